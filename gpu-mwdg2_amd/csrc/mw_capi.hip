@@ -15,6 +15,7 @@
 #include <mutex>
 #include <string>
 #include <sys/stat.h>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/mwdg2.h"
@@ -334,7 +335,7 @@ struct Ctx : CtxBase {
     for (uint8_t* p : {sig[0], sig[1], xflag, leaflev, preflag}) MW_HIP(hipMemsetAsync(p, 0, D + 4, stream));
     leaf = alloc<int>(N);
     for (int k = 0; k < 4; ++k) nbr[k] = alloc<int>(N);
-    tile_sums = alloc<int>(nblk(std::max(1, N / 4), EMIT_TILE) + 1);
+    tile_sums = alloc<int>(nblk(std::max(1, N / 4), EMIT_TILE_MIN) + 1);
     st = alloc<DevState<real>>(1);
     maxh2 = alloc<unsigned long long>(1);
     red = alloc<real>((size_t)5 * 2 * RED_SLOTS);
@@ -743,16 +744,37 @@ struct Ctx : CtxBase {
         timed("decode_level", [&] {
           if (mwm)
             launch_k((k_topdown_level<real, true>), dim3(g / WG), dim3(WG), 0, stream, st, hier[main_h], prev, nw,
-                     xflag, leaflev, L - 1, L, hc.epsilon, P.eps_extra_factor, cnt[1], tz);
+                     xflag, leaflev, L - 1, L, hc.epsilon, P.eps_extra_factor, cnt[1], tz, emit_tile());
           else
             launch_k((k_topdown_level<real, false>), dim3(g / WG), dim3(WG), 0, stream, st, hier[main_h], prev, nw,
-                     xflag, leaflev, L - 1, L, hc.epsilon, P.eps_extra_factor, cnt[1], tz);
+                     xflag, leaflev, L - 1, L, hc.epsilon, P.eps_extra_factor, cnt[1], tz, emit_tile());
         });
       }
     }
     return counted;
   }
-  int emit_tiles() const { return nblk(1 << (2 * (L - 1)), EMIT_TILE); }
+  // Nodes per emission tile: small grids need small tiles to have a
+  // work-group for every CU, large ones keep more of their neighbours inside
+  // a tile. us per launch with 64 / 256 / 1024 nodes: dam break 256^2 FP64
+  // 8.5 / 15 / 37, valley 1024^2 FP32 28 / 23 / 44, HWFV1 2048^2 (emit_write)
+  // 11 / 10 / 16, urban 4096^2 FP32 329 / 161 / 156; the single-group scan
+  // of the tiles' counts takes 4 us up to 4096 tiles and 24 us for 16384.
+  // The learned step's tiles hold whole level-6 units (one from
+  // max_ref_lvl 10 on).
+  int emit_tile() const {
+    const int t = L <= 9 ? 64 : (L <= 11 ? 256 : 1024);
+    return umode && L >= 10 ? 1 << (2 * (L - 1 - UNIT_LEVEL)) : t;
+  }
+  int emit_tiles() const { return nblk(1 << (2 * (L - 1)), emit_tile()); }
+  // f with the tile's node count as a constant
+  template <typename F>
+  void with_tile(F&& f) const {
+    switch (emit_tile()) {
+      case 64: f(std::integral_constant<int, 64>{}); break;
+      case 256: f(std::integral_constant<int, 256>{}); break;
+      default: f(std::integral_constant<int, 1024>{}); break;
+    }
+  }
   bool fuse_sweep1() const { return mwm && !hc.limitslopes; }
   // Leaf emission; with `sweep` (MWDG2 without limiter) the stage-1 sweep of
   // the emitted leaves runs in the same kernel.
@@ -763,19 +785,27 @@ struct Ctx : CtxBase {
     int* done = &st->done;
     int* nl = &st->n_leaves;
     if (!counted)
-      timed("emit_count", [&] { launch_k(k_emit_count, dim3(tiles), dim3(WG), 0, stream, done, leaflev, L, Q, tile_sums); });
+      timed("emit_count", [&] {
+        with_tile([&](auto T) {
+          launch_k(k_emit_count<T.value>, dim3(tiles), dim3(WG), 0, stream, done, leaflev, L, Q, tile_sums);
+        });
+      });
     timed("emit_scan", [&] { launch_k(k_emit_scan, dim3(1), dim3(1024), 0, stream, done, nl, tile_sums, tiles,
                                                   &st->clk_step, &st->mra_ticks); });
     if (sweep) {
       timed("emit_sweep1", [&] {
-        launch_k((k_emit_sweep1<real>), dim3(tiles), dim3(WG), 0, stream, st, P, leaflev, Q, tile_sums, leaf,
-                           nbr[0], nbr[1], nbr[2], nbr[3], hier[main_h], hier[main_h ^ 1], zh, wet[0]);
+        with_tile([&](auto T) {
+          launch_k((k_emit_sweep1<real, T.value>), dim3(tiles), dim3(WG), 0, stream, st, P, leaflev, Q, tile_sums,
+                   leaf, nbr[0], nbr[1], nbr[2], nbr[3], hier[main_h], hier[main_h ^ 1], zh, wet[0]);
+        });
       });
       return;
     }
     timed("emit_write", [&] {
-      launch_k(k_emit_write, dim3(tiles), dim3(WG), 0, stream, done, leaflev, L, Q, tile_sums, leaf, nbr[0],
-                         nbr[1], nbr[2], nbr[3], md, hc.xsz, hc.ysz);
+      with_tile([&](auto T) {
+        launch_k(k_emit_write<T.value>, dim3(tiles), dim3(WG), 0, stream, done, leaflev, L, Q, tile_sums, leaf,
+                 nbr[0], nbr[1], nbr[2], nbr[3], md, hc.xsz, hc.ysz);
+      });
     });
   }
   int sweep_g = 0;                            // work-groups of the leaf sweeps (0: the default)
@@ -1064,10 +1094,10 @@ struct Ctx : CtxBase {
     MW_HIP(hipMemsetAsync(utouch, 1, N_UNITS, stream));
   }
   // quiet units: the emission tiles of the fused stage-1 sweep hold whole
-  // units (max_ref_lvl <= 12, EMIT_TILE level-(L-1) items per tile)
+  // units (max_ref_lvl <= 12)
   void set_quiet_params() {
     P.dirty = learn ? dirty : nullptr;
-    static_assert(EMIT_TILE == 1 << (2 * (12 - 1 - UNIT_LEVEL)), "one unit per emission tile at max_ref_lvl 12");
+    static_assert(EMIT_TILE_MAX == 1 << (2 * (12 - 1 - UNIT_LEVEL)), "one unit per emission tile at max_ref_lvl 12");
     const bool q = learn && L <= 12 && fuse_sweep1();
     P.uquiet = q ? uquiet : nullptr;
     P.uwet = q ? uwet : nullptr;
@@ -1424,7 +1454,7 @@ struct Ctx : CtxBase {
     e.cnt_enc = cnt[0];
     e.cnt_dec = cnt[1];
     e.cnt_rescale = cnt[2];
-    e.tiles = emit_tiles();
+    e.tiles = nblk(1 << (2 * (L - 1)), EMIT_TILE_BATCH);
     e.Q = 1 << (2 * (L - 1));
     e.tile_sums = tile_sums;
     e.leaf = leaf;

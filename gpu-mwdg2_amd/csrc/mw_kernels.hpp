@@ -10,8 +10,12 @@ constexpr int WG = 256;          // work-group size (4 wave64s)
 // register cap that allows them); FP64 builds keep their registers (a cap
 // makes them spill).
 #define WAVES32(n) (sizeof(real) == 4 ? (n) : 1)
-constexpr int EMIT_ITEMS = 4;    // level-(L-1) nodes per thread in leaf emission
-constexpr int EMIT_TILE = WG * EMIT_ITEMS;
+// Level-(L-1) nodes of a leaf-emission tile (one work-group): the smallest and
+// the largest tile, and the tile of a batched ensemble pass.
+constexpr int EMIT_TILE_MIN = 64, EMIT_TILE_MAX = 1024, EMIT_TILE_BATCH = 1024;
+// Most level-6 units of the learned step that a tile of T nodes covers.
+template <int T>
+constexpr int EMIT_UNITS = T == EMIT_TILE_MIN ? 64 : (T == EMIT_TILE_MAX ? 1 : 4);
 constexpr int MAX_SRC = 4096;
 constexpr int RED_SLOTS = 4096;  // max work-groups of a leaf kernel (one reduction slot each)
 // Units of the learned step: level-6 nodes and their subtrees.

@@ -1,0 +1,48 @@
+"""Leaf emission over its tile sizes (64, 256 or 1024 level-(L-1) nodes per
+work-group): against the oracle, bit for bit, at the smallest grids (one part
+tile), on ragged DEMs and at the levels where the tile size changes; and the
+learned step's unit records with many units, several and one unit per tile."""
+import os
+
+import numpy as np
+import pytest
+
+import cases
+import parity_util
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("L,xsz,ysz,solver,prec", [
+    (2, 4, 3, "mwdg2", "f64"), (3, 8, 8, "hwfv1", "f32"), (4, 13, 16, "mwdg2", "f32"), (5, 32, 27, "hwfv1", "f64"),
+    (9, 401, 512, "mwdg2", "f32"), (10, 1024, 700, "hwfv1", "f32"), (10, 600, 1000, "mwdg2", "f64"),
+    (11, 1500, 1100, "mwdg2", "f32")])
+def test_emission_tiles(case_dir, L, xsz, ysz, solver, prec):
+    par = cases.random_case(os.path.join(str(case_dir), f"tile{L}{solver}{prec}"), L=L, seed=7 + L, xsz=xsz, ysz=ysz,
+                            solver=solver, manning=0.03, t_end=5.0, wet_frac=0.4,
+                            srcs=2 if L > 3 else 0, stage=2 if L > 3 else 0)
+    parity_util.run_pair(par, prec, steps=3)
+
+
+@pytest.mark.parametrize("L", [7, 8, 9, 10, 11])
+def test_learned_units_over_tiles(case_dir, L):
+    """With every unit frozen the learned step makes the plain step's tree;
+    its depths move from it by the rounding of the reconstructions it leaves
+    out, some 1e-16 of an elevation of 20 m per step (1e-9 m is far above
+    that and far below a wrong maximum, which changes the thresholds)."""
+    import mwdg2
+    from bench import finest_fields
+    par = cases.urban(os.path.join(str(case_dir), f"unit{L}"), L=L, t_end=100.0)
+    steps = 24
+    with mwdg2.Simulation(par, "f64") as ref:
+        ref.step(steps)
+        h_ref, leaves_ref = finest_fields(ref, L)[0], ref.get("leaves")
+        mx_ref = ref.counters()["maxes"]
+    with mwdg2.Mlp(3) as m, mwdg2.Simulation(par, "f64") as s:
+        s.set_learned(m, decide_every=8, full_every=32, threshold=2.0)
+        s.step(steps)
+        h, leaves = finest_fields(s, L)[0], s.get("leaves")
+        mx = s.counters()["maxes"]
+    assert np.array_equal(leaves, leaves_ref)
+    assert float(np.max(np.abs(h - h_ref))) <= 1e-9
+    assert np.allclose(mx, mx_ref, rtol=1e-9, atol=0)
