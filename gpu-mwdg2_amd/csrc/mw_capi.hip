@@ -335,7 +335,7 @@ struct Ctx : CtxBase {
     for (uint8_t* p : {sig[0], sig[1], xflag, leaflev, preflag}) MW_HIP(hipMemsetAsync(p, 0, D + 4, stream));
     leaf = alloc<int>(N);
     for (int k = 0; k < 4; ++k) nbr[k] = alloc<int>(N);
-    tile_sums = alloc<int>(nblk(std::max(1, N / 4), EMIT_TILE_MIN) + 1);
+    tile_sums = alloc<int>(nblk(std::max(1, N / 4), EMIT_TILE_MIN) + 4);   // read by fours
     st = alloc<DevState<real>>(1);
     maxh2 = alloc<unsigned long long>(1);
     red = alloc<real>((size_t)5 * 2 * RED_SLOTS);
@@ -604,19 +604,15 @@ struct Ctx : CtxBase {
   // with_sources: the prologue also applies the point sources (a step's
   // prologue; the single-stage calls launch k_point_sources on their own)
   // A step's prologue also zeroes the emission tiles' leaf counts, which the
-  // flat decode of level L-1 adds up (split_deepest).
+  // decode of level L-1 adds up (counts_tiles).
   void k_prologue_launch(bool with_sources = false) {
-    const bool zero = with_sources && split_deepest();
+    const bool zero = with_sources && counts_tiles();
     timed("prologue", [&] {
       launch_k((k_prologue<real>), dim3(1), dim3(PRO_WG), 0, stream, st, P, series(), sources(), red,
                2 * leaf_grid(), (with_sources && n_src) ? 1 : 0, hier[main_h], P.dirty,
                zero ? tile_sums : (int*)nullptr, zero ? emit_tiles() : 0);
     });
   }
-  // The deepest parent level L-1 of the encode and node level L-1 of the
-  // decode run as flat launches (one node per thread) beside their band
-  // kernels; plain step only (the learned step has its own band kernels).
-  bool split_deepest() const { return !lrn() && L - 1 > top_level(); }
   void k_sources_launch() {
     if (!n_src) return;
     timed("point_sources", [&] {
@@ -624,9 +620,10 @@ struct Ctx : CtxBase {
                P.dirty);
     });
   }
+  // Levels of the scale-only re-encode: 0 .. top_level() in one work-group,
+  // the rest in bands of at most 6 levels, deepest first; a band [lo, hi]
+  // runs one work-group per level-lo node.
   int top_level() const { return std::min(TOP_LEVEL, L - 1); }
-  // Levels top_level()+1 .. L-1 in bands of at most 6 levels, deepest first;
-  // a band [lo, hi] runs one work-group per level-lo node.
   std::vector<std::pair<int, int>> bands() const {
     std::vector<std::pair<int, int>> b;
     for (int hi = L - 1; hi > top_level();) {
@@ -636,8 +633,19 @@ struct Ctx : CtxBase {
     }
     return b;
   }
-  // FP32 MWDG2 runs the top levels' encode and decode as one kernel
-  bool fuse_top() const { return mwm && sizeof(real) == 4 && top_level() == TOP_LEVEL; }
+  // Levels of the encode and decode. From level 10 (4^10 nodes) on each level
+  // is a flat launch, one node per thread: there a level fills the chip, and
+  // a band's chain of barriers would hold most of its threads idle. Below,
+  // levels mra_lo .. mra_hi are one band launch whose work-groups have at most
+  // 256 nodes of the deepest level, one per thread, and levels 0 .. mra_top
+  // (at most 4: 341 nodes) one work-group. max_ref_lvl 12: flat 11 and 10,
+  // band 5-9, top 0-4; 10: band 5-9; 8: band 3-7, top 0-2. The learned step
+  // has its own kernels from level 6 on.
+  int mra_hi() const { return lrn() ? UNIT_LEVEL - 1 : std::min(L - 1, MRA_FLAT - 1); }
+  int mra_lo() const { return std::max(mra_hi() - (MRA_BAND - 1), 3); }
+  int mra_top() const { return std::min(mra_lo() - 1, L - 1); }
+  bool mra_band() const { return mra_lo() <= mra_hi(); }
+  bool counts_tiles() const { return !lrn() && mra_band(); }
   void encode_launch(bool skip_top = false) {
     uint8_t* prev = sig[cur];
     uint8_t* nw = sig[cur ^ 1];
@@ -654,64 +662,63 @@ struct Ctx : CtxBase {
                    nw, xflag, preflag, UNIT_LEVEL, L - 1, L, hc.epsilon, P.eps_extra_factor, cnt[0], ustat, P.dirty,
                    dm, D, full, ut);
       });
-    }
-    for (const auto& b : bands()) {
-      if (lrn()) break;
-      const int nwg = 1 << (2 * b.first);
-      int hi = b.second;
-      if (hi == L - 1 && split_deepest()) {        // level L-1 first, one parent per thread
-        const int g = 1 << (2 * (L - 1));
+    } else {
+      for (int level = L - 1; level > mra_hi(); --level) {
+        const int g = 1 << (2 * level);
         timed("encode_level", [&] {
           if (mwm)
             launch_k((k_encode_level<real, true>), dim3(g / WG), dim3(WG), 0, stream, st, hier[main_h], prev, nw,
-                     xflag, preflag, L - 1, L, hc.epsilon, P.eps_extra_factor, cnt[0]);
+                     xflag, preflag, level, L, hc.epsilon, P.eps_extra_factor, cnt[0]);
           else
             launch_k((k_encode_level<real, false>), dim3(g / WG), dim3(WG), 0, stream, st, hier[main_h], prev, nw,
-                     xflag, preflag, L - 1, L, hc.epsilon, P.eps_extra_factor, cnt[0]);
+                     xflag, preflag, level, L, hc.epsilon, P.eps_extra_factor, cnt[0]);
         });
-        --hi;
       }
-      if (hi < b.first) continue;
-      timed("encode", [&] {
+    }
+    if (mra_band())
+      timed(lrn() ? "encode_coarse" : "encode", [&] {
+        const int nwg = 1 << (2 * mra_lo());
         if (mwm)
           launch_k((k_encode_band<real, true>), dim3(nwg), dim3(WG), 0, stream, st, hier[main_h], prev, nw,
-                             xflag, preflag, b.first, hi, L, hc.epsilon, P.eps_extra_factor, cnt[0]);
+                             xflag, preflag, mra_lo(), mra_hi(), L, hc.epsilon, P.eps_extra_factor, cnt[0]);
         else
           launch_k((k_encode_band<real, false>), dim3(nwg), dim3(WG), 0, stream, st, hier[main_h], prev, nw,
-                             xflag, preflag, b.first, hi, L, hc.epsilon, P.eps_extra_factor, cnt[0]);
+                             xflag, preflag, mra_lo(), mra_hi(), L, hc.epsilon, P.eps_extra_factor, cnt[0]);
       });
-    }
-    if (skip_top) return;
-    timed("encode_top", [&] {
-      if (mwm)
-        launch_k((k_encode_top<real, true>), dim3(1), dim3(TOP_WG), 0, stream, st, hier[main_h], prev, nw, xflag,
-                           preflag, top_level(), L, hc.epsilon, P.eps_extra_factor, cnt[0]);
-      else
-        launch_k((k_encode_top<real, false>), dim3(1), dim3(TOP_WG), 0, stream, st, hier[main_h], prev, nw, xflag,
-                           preflag, top_level(), L, hc.epsilon, P.eps_extra_factor, cnt[0]);
-    });
+    if (!skip_top) top_launch(1);
   }
-  // Returns true when the flat decode of level L-1 also added up the
-  // emission tiles' leaf counts (count_tiles: the step's prologue zeroed them).
-  bool decode_launch(bool fused_top = false, bool count_tiles = false) {
+  // the coarse levels: mode 1 encode, 2 decode, 3 both
+  void top_launch(int mode) {
     uint8_t* prev = sig[cur];
     uint8_t* nw = sig[cur ^ 1];
-    if (fused_top) {
-      if constexpr (sizeof(real) == 4) {         // the node values of levels 0..5 fit the LDS in FP32
-        timed("top_mra", [&] {
-          launch_k((k_top_mra<real>), dim3(1), dim3(TOP_WG), 0, stream, st, hier[main_h], (const uint8_t*)prev, nw,
-                   xflag, (const uint8_t*)preflag, leaflev, top_level(), L, hc.epsilon, P.eps_extra_factor, cnt[0],
-                   cnt[1]);
-        });
-      }
-    } else timed("decode_top", [&] {
+    timed("top_mra", [&] {
+      const dim3 wg(top_threads(mra_top()));
       if (mwm)
-        launch_k((k_topdown_top<real, true>), dim3(1), dim3(TOP_WG), 0, stream, st, hier[main_h], prev, nw, xflag,
-                           leaflev, top_level(), L, hc.epsilon, P.eps_extra_factor, cnt[1]);
+        launch_k((k_top_mra<real, true>), dim3(1), wg, 0, stream, st, hier[main_h], (const uint8_t*)prev, nw, xflag,
+                 (const uint8_t*)preflag, leaflev, mra_top(), L, hc.epsilon, P.eps_extra_factor, cnt[0], cnt[1], mode);
       else
-        launch_k((k_topdown_top<real, false>), dim3(1), dim3(TOP_WG), 0, stream, st, hier[main_h], prev, nw, xflag,
-                           leaflev, top_level(), L, hc.epsilon, P.eps_extra_factor, cnt[1]);
+        launch_k((k_top_mra<real, false>), dim3(1), wg, 0, stream, st, hier[main_h], (const uint8_t*)prev, nw, xflag,
+                 (const uint8_t*)preflag, leaflev, mra_top(), L, hc.epsilon, P.eps_extra_factor, cnt[0], cnt[1], mode);
     });
+  }
+  // Returns true when the decode of level L-1 also added up the emission
+  // tiles' leaf counts (count_tiles: the step's prologue zeroed them).
+  bool decode_launch(bool with_encode = false, bool count_tiles = false) {
+    uint8_t* prev = sig[cur];
+    uint8_t* nw = sig[cur ^ 1];
+    top_launch(with_encode ? 3 : 2);
+    const bool counted = count_tiles && counts_tiles();
+    int* tz = counted ? tile_sums : nullptr;
+    if (mra_band())
+      timed(lrn() ? "decode_coarse" : "decode", [&] {
+        const int nwg = 1 << (2 * mra_lo());
+        if (mwm)
+          launch_k((k_topdown_band<real, true>), dim3(nwg), dim3(WG), 0, stream, st, hier[main_h], prev, nw,
+                   xflag, leaflev, mra_lo(), mra_hi(), L, hc.epsilon, P.eps_extra_factor, cnt[1], tz, emit_tile());
+        else
+          launch_k((k_topdown_band<real, false>), dim3(nwg), dim3(WG), 0, stream, st, hier[main_h], prev, nw,
+                   xflag, leaflev, mra_lo(), mra_hi(), L, hc.epsilon, P.eps_extra_factor, cnt[1], tz, emit_tile());
+      });
     if (lrn()) {
       timed("decode", [&] {
         launch_k((k_topdown_band_learn<real>), dim3(N_UNITS), dim3(WG), 0, stream, st, hier[main_h], prev, nw,
@@ -722,34 +729,17 @@ struct Ctx : CtxBase {
       });
       return false;
     }
-    const auto bs = bands();
-    bool counted = false;
-    for (auto it = bs.rbegin(); it != bs.rend(); ++it) {
-      const int nwg = 1 << (2 * it->first);
-      const bool split = it->second == L - 1 && split_deepest();
-      const int hi = split ? it->second - 1 : it->second;
-      if (hi >= it->first)
-        timed("decode", [&] {
-          if (mwm)
-            launch_k((k_topdown_band<real, true>), dim3(nwg), dim3(WG), 0, stream, st, hier[main_h], prev, nw,
-                     xflag, leaflev, it->first, hi, L, hc.epsilon, P.eps_extra_factor, cnt[1]);
-          else
-            launch_k((k_topdown_band<real, false>), dim3(nwg), dim3(WG), 0, stream, st, hier[main_h], prev, nw,
-                     xflag, leaflev, it->first, hi, L, hc.epsilon, P.eps_extra_factor, cnt[1]);
-        });
-      if (split) {                                  // level L-1, one node per thread; tile counts when zeroed
-        const int g = 1 << (2 * (L - 1));
-        int* tz = count_tiles ? tile_sums : nullptr;
-        counted = counted || count_tiles;
-        timed("decode_level", [&] {
-          if (mwm)
-            launch_k((k_topdown_level<real, true>), dim3(g / WG), dim3(WG), 0, stream, st, hier[main_h], prev, nw,
-                     xflag, leaflev, L - 1, L, hc.epsilon, P.eps_extra_factor, cnt[1], tz, emit_tile());
-          else
-            launch_k((k_topdown_level<real, false>), dim3(g / WG), dim3(WG), 0, stream, st, hier[main_h], prev, nw,
-                     xflag, leaflev, L - 1, L, hc.epsilon, P.eps_extra_factor, cnt[1], tz, emit_tile());
-        });
-      }
+    for (int level = mra_hi() + 1; level < L; ++level) {
+      const int g = 1 << (2 * level);
+      int* t = level == L - 1 ? tz : nullptr;
+      timed("decode_level", [&] {
+        if (mwm)
+          launch_k((k_topdown_level<real, true>), dim3(g / WG), dim3(WG), 0, stream, st, hier[main_h], prev, nw,
+                   xflag, leaflev, level, L, hc.epsilon, P.eps_extra_factor, cnt[1], t, emit_tile());
+        else
+          launch_k((k_topdown_level<real, false>), dim3(g / WG), dim3(WG), 0, stream, st, hier[main_h], prev, nw,
+                   xflag, leaflev, level, L, hc.epsilon, P.eps_extra_factor, cnt[1], t, emit_tile());
+      });
     }
     return counted;
   }
@@ -775,6 +765,9 @@ struct Ctx : CtxBase {
       default: f(std::integral_constant<int, 1024>{}); break;
     }
   }
+  EmitScan emit_scan_args(bool scanned) const {
+    return {tile_sums, scanned ? 1 : 0, &st->n_leaves, &st->clk_step, &st->mra_ticks};
+  }
   bool fuse_sweep1() const { return mwm && !hc.limitslopes; }
   // Leaf emission; with `sweep` (MWDG2 without limiter) the stage-1 sweep of
   // the emitted leaves runs in the same kernel.
@@ -790,12 +783,15 @@ struct Ctx : CtxBase {
           launch_k(k_emit_count<T.value>, dim3(tiles), dim3(WG), 0, stream, done, leaflev, L, Q, tile_sums);
         });
       });
-    timed("emit_scan", [&] { launch_k(k_emit_scan, dim3(1), dim3(1024), 0, stream, done, nl, tile_sums, tiles,
+    const bool scanned = tiles > EMIT_SELF_SCAN;
+    const EmitScan E = emit_scan_args(scanned);
+    if (scanned)
+      timed("emit_scan", [&] { launch_k(k_emit_scan, dim3(1), dim3(1024), 0, stream, done, nl, tile_sums, tiles,
                                                   &st->clk_step, &st->mra_ticks); });
     if (sweep) {
       timed("emit_sweep1", [&] {
         with_tile([&](auto T) {
-          launch_k((k_emit_sweep1<real, T.value>), dim3(tiles), dim3(WG), 0, stream, st, P, leaflev, Q, tile_sums,
+          launch_k((k_emit_sweep1<real, T.value>), dim3(tiles), dim3(WG), 0, stream, st, P, leaflev, Q, E,
                    leaf, nbr[0], nbr[1], nbr[2], nbr[3], hier[main_h], hier[main_h ^ 1], zh, wet[0]);
         });
       });
@@ -803,7 +799,7 @@ struct Ctx : CtxBase {
     }
     timed("emit_write", [&] {
       with_tile([&](auto T) {
-        launch_k(k_emit_write<T.value>, dim3(tiles), dim3(WG), 0, stream, done, leaflev, L, Q, tile_sums, leaf,
+        launch_k(k_emit_write<T.value>, dim3(tiles), dim3(WG), 0, stream, done, leaflev, L, Q, E, leaf,
                  nbr[0], nbr[1], nbr[2], nbr[3], md, hc.xsz, hc.ysz);
       });
     });
@@ -1130,9 +1126,8 @@ struct Ctx : CtxBase {
 
   bool l_full_step() const { return tr_x || !P.dirty || lstep % l_full == 0; }
   void rebuild(bool sweep = false) {
-    const bool ft = fuse_top();
-    encode_launch(ft);
-    const bool counted = decode_launch(ft, true);  // the step's prologue zeroed the tile sums
+    encode_launch(true);
+    const bool counted = decode_launch(true, true);  // the step's prologue zeroed the tile sums
     if (lrn() && P.uquiet)
       timed("learn", [&] {
         launch_k(k_unit_quiet, dim3(nblk(N_UNITS)), dim3(WG), 0, stream, (const uint8_t*)sig[cur ^ 1],
@@ -1457,6 +1452,7 @@ struct Ctx : CtxBase {
     e.tiles = nblk(1 << (2 * (L - 1)), EMIT_TILE_BATCH);
     e.Q = 1 << (2 * (L - 1));
     e.tile_sums = tile_sums;
+    e.scan = emit_scan_args(false);
     e.leaf = leaf;
     for (int k = 0; k < 4; ++k) e.nbr[k] = nbr[k];
     e.LL = leaves();
@@ -1464,12 +1460,17 @@ struct Ctx : CtxBase {
     e.W1 = wet[1];
     e.G = leaf_grid();
     e.src_blocks = n_src ? nblk(n_src) : 0;
+    e.mtop = mra_top();
+    e.mlo = mra_lo();
+    e.mhi = mra_hi();
     std::memcpy(out, &e, sizeof e);
     shape.max_tiles = std::max(shape.max_tiles, e.tiles);
     shape.max_g = std::max(shape.max_g, e.G);
     shape.max_src = std::max(shape.max_src, e.src_blocks);
     shape.units = std::max(shape.units, 1 << (2 * e.lo));
-    shape.fuse_top = fuse_top();
+    shape.mra_units = std::max(shape.mra_units, 1 << (2 * e.mlo));
+    shape.mra_top = std::max(shape.mra_top, e.mtop);
+    shape.max_level = std::max(shape.max_level, L - 1);
   }
   // One batched step of all scenarios of a table (this context only chooses
   // the precision): the pass order of one_step for the plain MWDG2 step.
@@ -1478,16 +1479,14 @@ struct Ctx : CtxBase {
     const unsigned S = (unsigned)sh.scenarios;
     hipLaunchKernelGGL(kb_prologue<real>, dim3(1, S), dim3(PRO_WG), 0, s, E);
     if (sh.max_src) hipLaunchKernelGGL(kb_point_sources<real>, dim3(sh.max_src, S), dim3(WG), 0, s, E);
-    hipLaunchKernelGGL(kb_encode_band<real>, dim3(sh.units, S), dim3(WG), 0, s, E);
-    if (sh.fuse_top) {
-      if constexpr (sizeof(real) == 4) hipLaunchKernelGGL(kb_top_mra<real>, dim3(1, S), dim3(TOP_WG), 0, s, E);
-    } else {
-      hipLaunchKernelGGL(kb_encode_top<real>, dim3(1, S), dim3(TOP_WG), 0, s, E);
-      hipLaunchKernelGGL(kb_topdown_top<real>, dim3(1, S), dim3(TOP_WG), 0, s, E);
-    }
-    hipLaunchKernelGGL(kb_topdown_band<real>, dim3(sh.units, S), dim3(WG), 0, s, E);
-    hipLaunchKernelGGL(kb_emit_count<real>, dim3(sh.max_tiles, S), dim3(WG), 0, s, E);
-    hipLaunchKernelGGL(kb_emit_scan<real>, dim3(1, S), dim3(1024), 0, s, E);
+    // the flat levels are launched for the scenarios that have them
+    for (int l = sh.max_level; l >= MRA_FLAT; --l)
+      hipLaunchKernelGGL(kb_encode_level<real>, dim3((1 << (2 * l)) / WG, S), dim3(WG), 0, s, E, l);
+    hipLaunchKernelGGL(kb_encode_band<real>, dim3(sh.mra_units, S), dim3(WG), 0, s, E);
+    hipLaunchKernelGGL(kb_top_mra<real>, dim3(1, S), dim3(top_threads(sh.mra_top)), 0, s, E);
+    hipLaunchKernelGGL(kb_topdown_band<real>, dim3(sh.mra_units, S), dim3(WG), 0, s, E);
+    for (int l = MRA_FLAT; l <= sh.max_level; ++l)
+      hipLaunchKernelGGL(kb_topdown_level<real>, dim3((1 << (2 * l)) / WG, S), dim3(WG), 0, s, E, l);
     hipLaunchKernelGGL(kb_emit_sweep1<real>, dim3(sh.max_tiles, S), dim3(WG), 0, s, E);
     hipLaunchKernelGGL(kb_wet1<real>, dim3(sh.max_g, S), dim3(WG), 0, s, E);
     hipLaunchKernelGGL(kb_encode_scale_band<real>, dim3(sh.units, S), dim3(WG), 0, s, E);

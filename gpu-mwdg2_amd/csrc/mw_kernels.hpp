@@ -10,9 +10,12 @@ constexpr int WG = 256;          // work-group size (4 wave64s)
 // register cap that allows them); FP64 builds keep their registers (a cap
 // makes them spill).
 #define WAVES32(n) (sizeof(real) == 4 ? (n) : 1)
+constexpr int MRA_FLAT = 10;     // encode and decode levels from this one on are flat launches
 // Level-(L-1) nodes of a leaf-emission tile (one work-group): the smallest and
 // the largest tile, and the tile of a batched ensemble pass.
 constexpr int EMIT_TILE_MIN = 64, EMIT_TILE_MAX = 1024, EMIT_TILE_BATCH = 1024;
+// Tiles whose leaf counts each emission work-group adds up itself.
+constexpr int EMIT_SELF_SCAN = 4096;
 // Most level-6 units of the learned step that a tile of T nodes covers.
 template <int T>
 constexpr int EMIT_UNITS = T == EMIT_TILE_MIN ? 64 : (T == EMIT_TILE_MAX ? 1 : 4);
@@ -37,8 +40,8 @@ struct DevState {
   int n_src;
   unsigned long long leaf_sum;    // leaves updated, summed over steps
   unsigned long long wet_sum[2];  // leaves of the wet lists of stage 1 and 2, summed over steps
-  int wet_n[2];                   // leaves on the wet lists of this step's stage 1 and 2
-  int coarse_leaves;              // set by the leaf emission when a leaf lies at a level <= TOP_LEVEL
+  alignas(128) int wet_n[2];      // leaves on the wet lists of this step's stage 1 and 2 (a line of their own)
+  alignas(128) int coarse_leaves; // set by the leaf emission when a leaf lies at a level <= TOP_LEVEL
   int save_count;                 // stage-output counter (classes/SaveInterval.h:47-56)
   int n_records;                  // stage-output rows written
   unsigned long long clk0;        // device wall clock at the first step's start
