@@ -123,7 +123,7 @@ struct CtxBase {
     // mode 2 times the leaf kernels and the MRA band kernels
     const bool update = !std::strncmp(name, "stage", 5) || !std::strncmp(name, "fv1", 3) ||
                         !std::strncmp(name, "sweep", 5) || !std::strncmp(name, "wet", 3) ||
-                        !std::strncmp(name, "emit_sweep", 10) || !std::strcmp(name, "encode") ||
+                        !std::strncmp(name, "emit_sweep", 10) || !std::strcmp(name, "emit_fv1") || !std::strcmp(name, "encode") ||
                         !std::strcmp(name, "decode") || !std::strcmp(name, "encode_scale") ||
                         !std::strcmp(name, "encode_level") || !std::strcmp(name, "decode_level");
     if (!profiling || (profiling == 2 && !update)) { launch(); return; }
@@ -769,6 +769,9 @@ struct Ctx : CtxBase {
     return {tile_sums, scanned ? 1 : 0, &st->n_leaves, &st->clk_step, &st->mra_ticks};
   }
   bool fuse_sweep1() const { return mwm && !hc.limitslopes; }
+  // HWFV1: the whole update in the leaf emission. Not with epsilon = 0, whose
+  // later steps read the neighbour lists of the one emission.
+  bool fuse_fv1() const { return !mwm && hc.epsilon > real(0) && emit_tile() == EMIT_TILE_MIN; }
   // Leaf emission; with `sweep` (MWDG2 without limiter) the stage-1 sweep of
   // the emitted leaves runs in the same kernel.
   // counted: the decode wrote the tiles' leaf counts already
@@ -788,6 +791,14 @@ struct Ctx : CtxBase {
     if (scanned)
       timed("emit_scan", [&] { launch_k(k_emit_scan, dim3(1), dim3(1024), 0, stream, done, nl, tile_sums, tiles,
                                                   &st->clk_step, &st->mra_ticks); });
+    if (sweep && !mwm) {
+      timed("emit_fv1", [&] {
+        launch_k((k_emit_fv1<real>), dim3(tiles), dim3(WG), 0, stream, st, P, leaflev, Q, E, leaf, hier[main_h],
+                 hier[main_h ^ 1], zh, red, 2 * leaf_grid());
+      });
+      main_h ^= 1;
+      return;
+    }
     if (sweep) {
       timed("emit_sweep1", [&] {
         with_tile([&](auto T) {
@@ -1149,10 +1160,10 @@ struct Ctx : CtxBase {
     const bool rb = hc.epsilon > real(0.0) || !issued_first;
     if (rb) {
       if (lrn()) learn_decide();
-      rebuild(fuse_sweep1());
+      rebuild(fuse_sweep1() || fuse_fv1());
       if (lrn()) learn_after();
     }
-    stage1_launch(rb && fuse_sweep1());
+    if (mwm || !fuse_fv1()) stage1_launch(rb && fuse_sweep1());
     if (mwm) {
       if (hc.epsilon > real(0.0)) encode_scale_launch(rb && fuse_sweep1());
       stage2_launch();
@@ -1644,8 +1655,9 @@ struct Ctx : CtxBase {
       if (name != "leaves") {
         const int k = name.size() == 4 ? name[3] - '0' : -1;
         if (k < 0 || k > 3) throw std::invalid_argument("unknown array " + name);
-        // the MWDG2 sweeps derive neighbours from the labels: materialise them
-        if (mwm && !hc.limitslopes && len > 0)
+        // the MWDG2 sweeps and the fused HWFV1 update derive neighbours from
+        // the labels: materialise them
+        if ((mwm ? !hc.limitslopes : fuse_fv1()) && len > 0)
           launch_k((k_fill_nbrs<real>), dim3(nblk(len)), dim3(WG), 0, stream, P, (const int*)&st->n_leaves,
                    (const int*)leaf, (const uint8_t*)leaflev, nbr[0], nbr[1], nbr[2], nbr[3]);
         dev = nbr[k];
