@@ -233,7 +233,7 @@ struct Ctx : CtxBase {
   int* tile_sums = nullptr;
   int *rev_z = nullptr, *rev_rm = nullptr;
   real* uprev = nullptr;
-  unsigned long long* maxh2 = nullptr;
+  unsigned long long* maxh = nullptr;         // limiter: per-work-group largest stage-1 depths (bit patterns)
   size_t Hp = 0;                              // node count rounded up to whole sibling groups
   real* xbuf = nullptr;                       // one coefficient as a plain array (parity transfers)
   real* red = nullptr;                        // [5][2 * leaf_grid()] next-step reduction slots
@@ -337,7 +337,7 @@ struct Ctx : CtxBase {
     for (int k = 0; k < 4; ++k) nbr[k] = alloc<int>(N);
     tile_sums = alloc<int>(nblk(std::max(1, N / 4), EMIT_TILE_MIN) + 4);   // read by fours
     st = alloc<DevState<real>>(1);
-    maxh2 = alloc<unsigned long long>(1);
+    maxh = alloc<unsigned long long>(RED_SLOTS);
     red = alloc<real>((size_t)5 * 2 * RED_SLOTS);
     {
       // neutral slots (dt +inf, maxima 0): kernels that do not write a slot leave it neutral
@@ -919,10 +919,10 @@ struct Ctx : CtxBase {
     timed(mwm ? "stage1" : "fv1", [&] {
       if (mwm)
         launch_k((k_stage1<real, true, true>), dim3(G), dim3(WG), 0, stream, st, P, leaves(), hier[main_h],
-                           hier[other], zh, uprev, red);
+                           hier[other], zh, uprev, red, maxh);
       else
         launch_k((k_stage1<real, false, false>), dim3(G), dim3(WG), 0, stream, st, P, leaves(),
-                           hier[main_h], hier[other], zh, uprev, red);
+                           hier[main_h], hier[other], zh, uprev, red, maxh);
     });
     if (!mwm) main_h = other;
   }
@@ -943,16 +943,18 @@ struct Ctx : CtxBase {
                          cnt[2], gated ? (const int*)&st->coarse_leaves : nullptr);
     });
   }
-  void stage2_launch() {
+  // alone: not after this step's stage 1 (whose kernel leaves the limiter's
+  // largest depths)
+  void stage2_launch(bool alone = false) {
     const int G = leaf_grid();
     if (hc.limitslopes) {
-      MW_HIP(hipMemsetAsync(maxh2, 0, sizeof(unsigned long long), stream));
-      timed("maxh2", [&] {
-        launch_k((k_maxh_stage2<real>), dim3(G), dim3(WG), 0, stream, st, P, leaves(), hier[1], zh, maxh2);
-      });
+      if (alone)
+        timed("maxh2", [&] {
+          launch_k((k_maxh_stage2<real>), dim3(G), dim3(WG), 0, stream, st, P, leaves(), hier[1], zh, maxh);
+        });
       timed("stage2", [&] {
         launch_k((k_stage2_limited<real>), dim3(G), dim3(WG), 0, stream, st, P, leaves(), hier[0], hier[1],
-                           zh, uprev, maxh2, red);
+                           zh, uprev, (const unsigned long long*)maxh, red);
       });
       return;
     }
@@ -1604,7 +1606,7 @@ struct Ctx : CtxBase {
     else if (s == "swap_masks") cur ^= 1;
     else if (s == "stage1" || s == "fv1") { reset_wet_list(0); stage1_launch(); }
     else if (s == "encode_scale") encode_scale_launch();
-    else if (s == "stage2") { reset_wet_list(1); stage2_launch(); }
+    else if (s == "stage2") { reset_wet_list(1); stage2_launch(true); }
     else if (s == "mark_first_issued") issued_first = true;
     else throw std::invalid_argument("unknown stage " + s);
     MW_HIP(hipGetLastError());

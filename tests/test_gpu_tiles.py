@@ -46,3 +46,31 @@ def test_learned_units_over_tiles(case_dir, L):
     assert np.array_equal(leaves, leaves_ref)
     assert float(np.max(np.abs(h - h_ref))) <= 1e-9
     assert np.allclose(mx, mx_ref, rtol=1e-9, atol=0)
+
+
+@pytest.mark.parametrize("L,solver,prec,limit", [
+    (3, "mwdg2", "f64", False), (5, "hwfv1", "f32", False), (8, "mwdg2", "f32", False), (8, "hwfv1", "f64", False),
+    (7, "mwdg2", "f64", True), (10, "mwdg2", "f32", True)])
+def test_single_stages_make_the_step(case_dir, L, solver, prec, limit):
+    """The stages called one by one (encode and decode apart, the limiter's
+    largest depth taken from B) give what whole steps give, bit for bit."""
+    import mwdg2
+    par = cases.random_case(os.path.join(str(case_dir), f"stg{L}{solver}{prec}{limit}"), L=L, seed=3 + L,
+                            solver=solver, manning=0.03, t_end=50.0, srcs=3 if L > 3 else 0)
+    if limit:
+        with open(par, "a") as f:
+            f.write("limitslopes\ntol_Krivo     1\n")
+    stages = ["prologue", "point_sources", "encode", "decode", "emit", "swap_masks"]
+    stages += ["stage1", "encode_scale", "stage2"] if solver == "mwdg2" else ["fv1"]
+    with mwdg2.Simulation(par, prec) as a, mwdg2.Simulation(par, prec) as b:
+        a.step(3)
+        for _ in range(3):
+            for name in stages:
+                b.stage(name)
+        ca, cb = a.counters(), b.counters()
+        assert ca["time"] == cb["time"] and ca["dt_next"] == cb["dt_next"] and ca["n_leaves"] == cb["n_leaves"]
+        leaves = a.get("leaves")
+        assert np.array_equal(leaves, b.get("leaves"))
+        assert np.array_equal(a.get("sig")[3:], b.get("sig")[3:])
+        for c in ("eta0", "qx0", "qy0") + (("eta1x", "qx1y", "qy1x") if solver == "mwdg2" else ()):
+            assert np.array_equal(a.get("A." + c)[leaves], b.get("A." + c)[leaves]), c
