@@ -238,6 +238,7 @@ struct Ctx : CtxBase {
   real* xbuf = nullptr;                       // one coefficient as a plain array (parity transfers)
   real* red = nullptr;                        // [5][2 * leaf_grid()] next-step reduction slots
   WetList wet[2]{};                           // wet-leaf lists of the two MWDG2 stages
+  int* list_n = nullptr;                      // their counters
   int n_stage = 0;                            // gauges (stage points)
   int* stage_codes = nullptr;
   real* rec = nullptr;                        // stage-output rows: time, depths, elevations, velocities
@@ -610,7 +611,7 @@ struct Ctx : CtxBase {
     timed("prologue", [&] {
       launch_k((k_prologue<real>), dim3(1), dim3(PRO_WG), 0, stream, st, P, series(), sources(), red,
                2 * leaf_grid(), (with_sources && n_src) ? 1 : 0, hier[main_h], P.dirty,
-               zero ? tile_sums : (int*)nullptr, zero ? emit_tiles() : 0);
+               zero ? tile_sums : (int*)nullptr, zero ? emit_tiles() : 0, list_n);
     });
   }
   void k_sources_launch() {
@@ -830,9 +831,8 @@ struct Ctx : CtxBase {
   int leaf_grid() const { return sweep_g ? sweep_g : default_sweep_groups(); }
   int sweep_groups() const override { return leaf_grid(); }
   // The sweeps' work-group count (a multiple of 8, 8 .. 4096). The per-group
-  // reduction slots of the last step are folded into the new layout and the
-  // wet-list regions are re-sized; results do not depend on it (exact
-  // min/max reductions, per-leaf updates).
+  // reduction slots of the last step are folded into the new layout; results
+  // do not depend on it (exact min/max reductions, per-leaf updates).
   void set_sweep_groups(int g) override {
     not_in_ensemble("set_sweep_groups");
     if (!mwm || hc.limitslopes) throw std::invalid_argument("sweep groups apply to the MWDG2 sweeps without limiter");
@@ -853,7 +853,6 @@ struct Ctx : CtxBase {
     }
     MW_HIP(hipMemcpy(red, nw.data(), sizeof(real) * nw.size(), hipMemcpyHostToDevice));
     sweep_g = g;
-    alloc_wet_lists();
     MW_HIP(hipStreamSynchronize(stream));
   }
   void release(void* p) {
@@ -861,19 +860,23 @@ struct Ctx : CtxBase {
     allocs.erase(std::remove(allocs.begin(), allocs.end(), p), allocs.end());
     (void)hipFree(p);
   }
-  // wet-leaf lists of the two stages: at most one entry per finest cell,
-  // counters in the device state (reset by the prologue)
+  // The wet lists: a region holds the leaves of its share of the emission's
+  // tiles (of any tile size) or of the sweeps' (256 leaves). Small grids, with
+  // few appends, have 8 regions.
   void alloc_wet_lists() {
-    for (int q = 0; q < 2; ++q) {
-      if (!wet[q].list) wet[q].list = alloc<int>(N);
-      wet[q].n = &st->wet_n[q];
-      wet[q].sum = &st->wet_sum[q];
-      wet[q].cap = N;
-    }
+    if (list_n) return;
+    const int R = L <= 9 ? 8 : LIST_REGIONS;
+    long long cap = 0;
+    for (int t : {EMIT_TILE_MIN, 256, EMIT_TILE_MAX})             // the smallest hold 256 leaves, as the sweeps'
+      cap = std::max(cap, (long long)nblk(nblk(std::max(1, N / 4), t), R) * 4 * t);
+    list_n = alloc<int>(2 * LIST_REGIONS * LIST_PAD);
+    MW_HIP(hipMemsetAsync(list_n, 0, sizeof(int) * 2 * LIST_REGIONS * LIST_PAD, stream));
+    for (int q = 0; q < 2; ++q)
+      wet[q] = {alloc<int>((size_t)R * cap), list_n + q * LIST_REGIONS * LIST_PAD, &st->wet_sum[q], (int)cap, R};
   }
   // a single stage run without the prologue starts its wet list afresh
   void reset_wet_list(int q) {
-    if (mwm && !hc.limitslopes) MW_HIP(hipMemsetAsync(&st->wet_n[q], 0, sizeof(int), stream));
+    if (mwm && !hc.limitslopes) MW_HIP(hipMemsetAsync(wet[q].n, 0, sizeof(int) * LIST_REGIONS * LIST_PAD, stream));
   }
   void check_graphable() const override {
     if (!mwm || hc.limitslopes) throw std::invalid_argument("ensembles run the MWDG2 step without limiter");
@@ -1471,6 +1474,7 @@ struct Ctx : CtxBase {
     e.LL = leaves();
     e.W0 = wet[0];
     e.W1 = wet[1];
+    e.list_n = list_n;
     e.G = leaf_grid();
     e.src_blocks = n_src ? nblk(n_src) : 0;
     e.mtop = mra_top();

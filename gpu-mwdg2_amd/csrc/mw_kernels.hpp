@@ -14,6 +14,9 @@ constexpr int MRA_FLAT = 10;     // encode and decode levels from this one on ar
 // Level-(L-1) nodes of a leaf-emission tile (one work-group): the smallest and
 // the largest tile, and the tile of a batched ensemble pass.
 constexpr int EMIT_TILE_MIN = 64, EMIT_TILE_MAX = 1024, EMIT_TILE_BATCH = 1024;
+// Wet lists: regions at most, and ints between two regions' counters (a
+// 128-byte line each).
+constexpr int LIST_REGIONS = 64, LIST_PAD = 32;
 // Tiles whose leaf counts each emission work-group adds up itself.
 constexpr int EMIT_SELF_SCAN = 4096;
 // Most level-6 units of the learned step that a tile of T nodes covers.
@@ -40,7 +43,6 @@ struct DevState {
   int n_src;
   unsigned long long leaf_sum;    // leaves updated, summed over steps
   unsigned long long wet_sum[2];  // leaves of the wet lists of stage 1 and 2, summed over steps
-  alignas(128) int wet_n[2];      // leaves on the wet lists of this step's stage 1 and 2 (a line of their own)
   alignas(128) int coarse_leaves; // set by the leaf emission when a leaf lies at a level <= TOP_LEVEL
   int save_count;                 // stage-output counter (classes/SaveInterval.h:47-56)
   int n_records;                  // stage-output rows written

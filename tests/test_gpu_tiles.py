@@ -74,3 +74,14 @@ def test_single_stages_make_the_step(case_dir, L, solver, prec, limit):
         assert np.array_equal(a.get("sig")[3:], b.get("sig")[3:])
         for c in ("eta0", "qx0", "qy0") + (("eta1x", "qx1y", "qy1x") if solver == "mwdg2" else ()):
             assert np.array_equal(a.get("A." + c)[leaves], b.get("A." + c)[leaves]), c
+
+
+@pytest.mark.parametrize("L,eps", [(4, 1e-3), (9, 1e-3), (9, 0.0), (10, 0.0), (11, 1e-4)])
+def test_wet_lists_full_and_in_one_part(case_dir, L, eps):
+    """Every leaf wet (each region of the wet lists holds all its share), from
+    the emission (epsilon > 0) and from the sweeps (epsilon 0); at the largest
+    level a small DEM in one corner of the mesh, so that few regions hold it all."""
+    side = {11: 200}.get(L)
+    par = cases.random_case(os.path.join(str(case_dir), f"full{L}{eps}"), L=L, seed=41 + L, eps=eps, manning=0.03,
+                            t_end=50.0, wet_frac=1.0, xsz=side, ysz=side)
+    parity_util.run_pair(par, "f32", steps=3)
