@@ -125,6 +125,7 @@ struct CtxBase {
                         !std::strncmp(name, "sweep", 5) || !std::strncmp(name, "wet", 3) ||
                         !std::strncmp(name, "emit_sweep", 10) || !std::strcmp(name, "emit_fv1") || !std::strcmp(name, "encode") ||
                         !std::strcmp(name, "decode") || !std::strcmp(name, "encode_scale") ||
+                        !std::strcmp(name, "encode_scale_level") ||
                         !std::strcmp(name, "encode_level") || !std::strcmp(name, "decode_level");
     if (!profiling || (profiling == 2 && !update)) { launch(); return; }
     hipEvent_t a = ev(), b = ev();
@@ -621,30 +622,25 @@ struct Ctx : CtxBase {
                P.dirty);
     });
   }
-  // Levels of the scale-only re-encode: 0 .. top_level() in one work-group,
-  // the rest in bands of at most 6 levels, deepest first; a band [lo, hi]
-  // runs one work-group per level-lo node.
-  int top_level() const { return std::min(TOP_LEVEL, L - 1); }
-  std::vector<std::pair<int, int>> bands() const {
-    std::vector<std::pair<int, int>> b;
-    for (int hi = L - 1; hi > top_level();) {
-      const int lo = std::max(top_level() + 1, hi - 5);
-      b.push_back({lo, hi});
-      hi = lo - 1;
-    }
-    return b;
-  }
-  // Levels of the encode and decode. From level 10 (4^10 nodes) on each level
+  // Levels of the encode, the decode and the stage-1 re-encode. From level 10 (4^10 nodes) on each level
   // is a flat launch, one node per thread: there a level fills the chip, and
   // a band's chain of barriers would hold most of its threads idle. Below,
   // levels mra_lo .. mra_hi are one band launch whose work-groups have at most
   // 256 nodes of the deepest level, one per thread, and levels 0 .. mra_top
   // (at most 4: 341 nodes) one work-group. max_ref_lvl 12: flat 11 and 10,
   // band 5-9, top 0-4; 10: band 5-9; 8: band 3-7, top 0-2. The learned step
-  // has its own kernels from level 6 on.
-  int mra_hi() const { return lrn() ? UNIT_LEVEL - 1 : std::min(L - 1, MRA_FLAT - 1); }
-  int mra_lo() const { return std::max(mra_hi() - (MRA_BAND - 1), 3); }
-  int mra_top() const { return std::min(mra_lo() - 1, L - 1); }
+  // has its own encode and decode kernels from level 6 on.
+  struct Levels {
+    int lo, hi, top;
+    bool band() const { return lo <= hi; }
+  };
+  Levels levels(int deepest) const {
+    const int hi = std::min(deepest, MRA_FLAT - 1), lo = std::max(hi - (MRA_BAND - 1), 3);
+    return {lo, hi, std::min(lo - 1, L - 1)};
+  }
+  int mra_hi() const { return levels(lrn() ? UNIT_LEVEL - 1 : L - 1).hi; }
+  int mra_lo() const { return levels(lrn() ? UNIT_LEVEL - 1 : L - 1).lo; }
+  int mra_top() const { return levels(lrn() ? UNIT_LEVEL - 1 : L - 1).top; }
   bool mra_band() const { return mra_lo() <= mra_hi(); }
   bool counts_tiles() const { return !lrn() && mra_band(); }
   void encode_launch(bool skip_top = false) {
@@ -932,18 +928,22 @@ struct Ctx : CtxBase {
   // gated: the leaf emission of this step ran in k_emit_sweep1, which marks
   // leaves at levels <= TOP_LEVEL (the top re-encode is skipped without them)
   void encode_scale_launch(bool gated = false) {
-    for (const auto& b : bands()) {
-      const int nwg = 1 << (2 * b.first);
-      timed("encode_scale", [&] {
-        // quiet units (one band of level-6 units) keep their stage-1 parents
-        const uint8_t* q = (P.uquiet && b.first == UNIT_LEVEL) ? P.uquiet : nullptr;
-        launch_k((k_encode_scale_band<real>), dim3(nwg), dim3(WG), 0, stream, st, hier[1], sig[cur], b.first,
-                           b.second, cnt[2], q);
+    const uint8_t* q = P.uquiet;                    // quiet units keep their stage-1 parents
+    const int* gate = gated ? (const int*)&st->coarse_leaves : nullptr;
+    const Levels v = levels(L - 1);
+    for (int level = L - 1; level > v.hi; --level)
+      timed("encode_scale_level", [&] {
+        launch_k((k_scale_level<real>), dim3((1 << (2 * level)) / WG), dim3(WG), 0, stream, st, hier[1],
+                 (const uint8_t*)sig[cur], level, cnt[2], q);
       });
-    }
+    if (v.band())
+      timed("encode_scale", [&] {
+        launch_k((k_scale_band<real>), dim3(1 << (2 * v.lo)), dim3(WG), 0, stream, st, hier[1],
+                 (const uint8_t*)sig[cur], v.lo, v.hi, cnt[2], q, gate);
+      });
     timed("encode_scale_top", [&] {
-      launch_k((k_encode_scale_top<real>), dim3(1), dim3(TOP_WG), 0, stream, st, hier[1], sig[cur], top_level(),
-                         cnt[2], gated ? (const int*)&st->coarse_leaves : nullptr);
+      launch_k((k_scale_top<real>), dim3(1), dim3(top_threads(v.top)), 0, stream, st, hier[1],
+               (const uint8_t*)sig[cur], v.top, cnt[2], gate);
     });
   }
   // alone: not after this step's stage 1 (whose kernel leaves the limiter's
@@ -976,9 +976,8 @@ struct Ctx : CtxBase {
   void learn_alloc() {
     if (!mwm || !(hc.epsilon > real(0)) || hc.limitslopes)
       throw std::invalid_argument("learned refinement needs the MWDG2 solver without slope limiter and epsilon > 0");
-    const auto b = bands();
-    if (b.size() != 1 || b[0].first != UNIT_LEVEL || b[0].second != L - 1)
-      throw std::invalid_argument("learned refinement needs 7 <= max_ref_lvl <= 12 (one MRA band of level-6 units)");
+    if (L <= UNIT_LEVEL || L > 12)
+      throw std::invalid_argument("learned refinement needs 7 <= max_ref_lvl <= 12");
     if (umode) return;
     umode = alloc<uint8_t>(N_UNITS);
     uchg = alloc<uint8_t>(N_UNITS);
@@ -1433,7 +1432,7 @@ struct Ctx : CtxBase {
   // A scenario of a batched ensemble: the plain MWDG2 step without limiter,
   // epsilon > 0, one MRA band of level-6 units, no recording.
   bool batchable() const override {
-    return mwm && !hc.limitslopes && hc.epsilon > real(0.0) && L >= 7 && L <= 12 && bands().size() == 1 &&
+    return mwm && !hc.limitslopes && hc.epsilon > real(0.0) && L >= 7 && L <= 12 &&
            !rec && !cum && !learn && !tr_x && !profiling;
   }
   size_t batch_args_size() const override { return sizeof(EnsArgs<real>); }
@@ -1456,9 +1455,6 @@ struct Ctx : CtxBase {
     e.preflag = preflag;
     e.leaflev = leaflev;
     e.L = L;
-    e.top = top_level();
-    e.lo = bands()[0].first;
-    e.hi = bands()[0].second;
     e.eps = hc.epsilon;
     e.xfac = P.eps_extra_factor;
     e.dx = hc.dx;
@@ -1484,7 +1480,6 @@ struct Ctx : CtxBase {
     shape.max_tiles = std::max(shape.max_tiles, e.tiles);
     shape.max_g = std::max(shape.max_g, e.G);
     shape.max_src = std::max(shape.max_src, e.src_blocks);
-    shape.units = std::max(shape.units, 1 << (2 * e.lo));
     shape.mra_units = std::max(shape.mra_units, 1 << (2 * e.mlo));
     shape.mra_top = std::max(shape.mra_top, e.mtop);
     shape.max_level = std::max(shape.max_level, L - 1);
@@ -1506,8 +1501,10 @@ struct Ctx : CtxBase {
       hipLaunchKernelGGL(kb_topdown_level<real>, dim3((1 << (2 * l)) / WG, S), dim3(WG), 0, s, E, l);
     hipLaunchKernelGGL(kb_emit_sweep1<real>, dim3(sh.max_tiles, S), dim3(WG), 0, s, E);
     hipLaunchKernelGGL(kb_wet1<real>, dim3(sh.max_g, S), dim3(WG), 0, s, E);
-    hipLaunchKernelGGL(kb_encode_scale_band<real>, dim3(sh.units, S), dim3(WG), 0, s, E);
-    hipLaunchKernelGGL(kb_encode_scale_top<real>, dim3(1, S), dim3(TOP_WG), 0, s, E);
+    for (int l = sh.max_level; l >= MRA_FLAT; --l)
+      hipLaunchKernelGGL(kb_scale_level<real>, dim3((1 << (2 * l)) / WG, S), dim3(WG), 0, s, E, l);
+    hipLaunchKernelGGL(kb_scale_band<real>, dim3(sh.mra_units, S), dim3(WG), 0, s, E);
+    hipLaunchKernelGGL(kb_scale_top<real>, dim3(1, S), dim3(top_threads(sh.mra_top)), 0, s, E);
     hipLaunchKernelGGL(kb_sweep2<real>, dim3(sh.max_g, S), dim3(WG), 0, s, E);
     hipLaunchKernelGGL(kb_wet2<real>, dim3(sh.max_g, S), dim3(WG), 0, s, E);
     MW_HIP(hipGetLastError());
