@@ -698,6 +698,15 @@ struct Ctx : CtxBase {
                  (const uint8_t*)preflag, leaflev, mra_top(), L, hc.epsilon, P.eps_extra_factor, cnt[0], cnt[1], mode);
     });
   }
+  // HWFV1's whole encode and decode in one work-group
+  bool hw_tree() const { return !mwm && !lrn() && mra_band() && L <= HW_TREE_LEVELS; }
+  void hw_tree_launch() {
+    timed("hw_tree", [&] {
+      launch_k((k_hw_tree<real>), dim3(1), dim3(1 << (2 * (L - 1))), 0, stream, st, hier[main_h],
+               (const uint8_t*)sig[cur], sig[cur ^ 1], xflag, (const uint8_t*)preflag, leaflev, L, hc.epsilon,
+               P.eps_extra_factor, cnt[0], cnt[1], tile_sums, emit_tile());
+    });
+  }
   // Returns true when the decode of level L-1 also added up the emission
   // tiles' leaf counts (count_tiles: the step's prologue zeroed them).
   bool decode_launch(bool with_encode = false, bool count_tiles = false) {
@@ -1141,8 +1150,13 @@ struct Ctx : CtxBase {
 
   bool l_full_step() const { return tr_x || !P.dirty || lstep % l_full == 0; }
   void rebuild(bool sweep = false) {
-    encode_launch(true);
-    const bool counted = decode_launch(true, true);  // the step's prologue zeroed the tile sums
+    bool counted = hw_tree();                        // the step's prologue zeroed the tile sums
+    if (counted) {
+      hw_tree_launch();
+    } else {
+      encode_launch(true);
+      counted = decode_launch(true, true);
+    }
     if (lrn() && P.uquiet)
       timed("learn", [&] {
         launch_k(k_unit_quiet, dim3(nblk(N_UNITS)), dim3(WG), 0, stream, (const uint8_t*)sig[cur ^ 1],

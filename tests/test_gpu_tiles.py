@@ -85,3 +85,26 @@ def test_wet_lists_full_and_in_one_part(case_dir, L, eps):
     par = cases.random_case(os.path.join(str(case_dir), f"full{L}{eps}"), L=L, seed=41 + L, eps=eps, manning=0.03,
                             t_end=50.0, wet_frac=1.0, xsz=side, ysz=side)
     parity_util.run_pair(par, "f32", steps=3)
+
+
+@pytest.mark.parametrize("L,prec", [(4, "f32"), (4, "f64"), (5, "f32"), (6, "f32"), (6, "f64"), (7, "f32")])
+def test_hwfv1_small_trees(case_dir, L, prec):
+    """HWFV1's whole tree in one work-group (4 to 6 parent levels) and one level
+    above it: the oracle's, bit for bit, on a full grid over enough steps for the
+    tree to change; and the stages apart make the same."""
+    import mwdg2
+    par = cases.random_case(os.path.join(str(case_dir), f"hw{L}{prec}"), L=L, seed=50 + L, solver="hwfv1",
+                            manning=0.03, t_end=50.0, wet_frac=0.5, srcs=2, stage=2)
+    parity_util.run_pair(par, prec, steps=6)
+    with mwdg2.Simulation(par, prec) as a, mwdg2.Simulation(par, prec) as b:
+        a.step(4)
+        for _ in range(4):
+            for name in ["prologue", "point_sources", "encode", "decode", "emit", "swap_masks", "fv1"]:
+                b.stage(name)
+        ca, cb = a.counters(), b.counters()
+        assert ca["time"] == cb["time"] and ca["dt_next"] == cb["dt_next"] and ca["n_leaves"] == cb["n_leaves"]
+        leaves = a.get("leaves")
+        assert np.array_equal(leaves, b.get("leaves"))
+        assert np.array_equal(a.get("sig")[3:], b.get("sig")[3:])
+        for c in ("eta0", "qx0", "qy0"):
+            assert np.array_equal(a.get("A." + c), b.get("A." + c)), c
