@@ -100,11 +100,11 @@ def kernel_bytes(s: int, L: int, leaves: int, wet1: int, wet2: int, p_enc: int =
     {0, 1x, 1y}); 9 of them (not z) are written. Stage 1: the sweep reads all
     leaves and writes the dry ones (and a 4-byte list entry per wet leaf); the
     wet kernel reads and writes the wet leaves. Stage 2 likewise, where a leaf
-    also reads its 9 stage-start coefficients from A. The band kernels (parent
-    levels 6 .. L-1, `steps` launches each): an encoded parent reads its 4
+    also reads its 9 stage-start coefficients from A. The tree passes (flat
+    and band kernels together, `steps` passes each): an encoded parent reads its 4
     children's 9 coefficients and writes its own 9; a decoded parent reads
     and writes its children's 36; a re-encoded (stage-1) parent reads 36 and
-    writes 9; plus one byte per band node for each mask read or written
+    writes 9; plus one byte per node from level 6 down for each mask read or written
     (encode: previous tree and preflags in, new tree and extra-significance
     flags out; decode: three in, tree and leaf labels out; re-encode: the
     tree in).
@@ -158,11 +158,12 @@ def measured_traffic(kernel: str):
     """HBM bytes per dispatch of `kernel` (read + write) from the committed
     rocprofv3 FETCH_SIZE / WRITE_SIZE summary of this workload, each counter
     scaled by its reading for a 1 GiB copy kernel; None if not recorded."""
-    # the encode and decode passes: their band kernel and their flat kernel
-    # of level L-1, one launch each per step
-    names = {"encode": ["k_encode_band<float,true>", "k_encode_level<float,true>"],
-             "decode": ["k_topdown_band<float,true>", "k_topdown_level<float,true>"],
-             "encode_scale": ["k_encode_scale_band<float>"]}.get(kernel, [f"k_{kernel}<float>"])
+    # the tree passes at max_ref_lvl 12: a band kernel and the flat kernel of
+    # levels 10 and 11, two launches a step
+    names = {"encode": {"k_encode_band<float,true>": 1, "k_encode_level<float,true>": 2},
+             "decode": {"k_topdown_band<float,true>": 1, "k_topdown_level<float,true>": 2},
+             "encode_scale": {"k_scale_band<float>": 1, "k_scale_level<float>": 2},
+             "emit_sweep1": {"k_emit_sweep1<float,1024>": 1}}.get(kernel, {f"k_{kernel}<float>": 1})
     path = os.path.join(ROOT, "profiles", "hbm_traffic_urban_L12.txt")
     total, found = 0, False
     try:
@@ -170,7 +171,7 @@ def measured_traffic(kernel: str):
             for line in f:
                 parts = line.split()
                 if len(parts) == 4 and parts[0] == "traffic" and parts[1] in names:
-                    total += int(float(parts[2]) + float(parts[3]))
+                    total += names[parts[1]] * int(float(parts[2]) + float(parts[3]))
                     found = True
     except OSError:
         pass
@@ -607,10 +608,11 @@ def main():
     prof = sim.profile_read()
     sim.profile(0)
     c2 = sim.counters()
-    # the encode and decode passes are a band kernel and a flat kernel of
-    # level L-1 each: timed together, one pass per step
+    # the tree passes are a band kernel and flat kernels of the levels below
+    # it: timed together, one pass per step
     passes = dict(prof)
-    for band, flat in (("encode", "encode_level"), ("decode", "decode_level")):
+    for band, flat in (("encode", "encode_level"), ("decode", "decode_level"),
+                       ("encode_scale", "encode_scale_level")):
         if flat in passes:
             n, ms = passes.pop(flat)
             passes[band] = (passes[band][0], passes[band][1] + ms) if band in passes else (n, ms)
