@@ -231,6 +231,7 @@ struct Ctx : CtxBase {
   uint8_t *xflag = nullptr, *leaflev = nullptr, *preflag = nullptr;
   int* leaf = nullptr;
   int* nbr[4] = {nullptr, nullptr, nullptr, nullptr};
+  bool nbr_behind = false;                    // HWFV1: the last leaf list's neighbour lists are not written yet
   int* tile_sums = nullptr;
   int *rev_z = nullptr, *rev_rm = nullptr;
   real* uprev = nullptr;
@@ -1557,6 +1558,7 @@ struct Ctx : CtxBase {
   void reconcile(const DevState<real>& s) {
     const long long performed = (long long)s.steps - dev_steps_at_sync;
     const long long wasted = issued_since_sync - performed;
+    if (fuse_fv1() && std::min(performed, issued_since_sync) > 0) nbr_behind = true;
     issued_since_sync = 0;
     dev_steps_at_sync = s.steps;
     if (wasted <= 0 || in_ensemble) return;
@@ -1567,6 +1569,24 @@ struct Ctx : CtxBase {
       issued_first = false;
     }
     if (!mwm) main_h ^= (int)(wasted & 1);
+  }
+
+  // The fused HWFV1 update (k_emit_fv1) uses a leaf's neighbours where it
+  // derives them and leaves the lists unwritten (at 512^2 the stores cost 1 us
+  // of a 52 us step). They follow from the leaf list and its labels, so they
+  // are written here, before a call that reads them or changes either.
+  void write_nbrs() {
+    if (mwm) return;
+    const DevState<real> s = read_state();
+    if (!nbr_behind) return;
+    nbr_behind = false;
+    fill_nbrs(s.n_leaves);
+  }
+  void fill_nbrs(int n) {
+    if (n > 0)
+      launch_k((k_fill_nbrs<real>), dim3(nblk(n)), dim3(WG), 0, stream, P, (const int*)&st->n_leaves,
+               (const int*)leaf, (const uint8_t*)leaflev, nbr[0], nbr[1], nbr[2], nbr[3]);
+    MW_HIP(hipGetLastError());
   }
 
   // minimum over the reduction slots written by the last update kernel
@@ -1613,6 +1633,7 @@ struct Ctx : CtxBase {
     if (learn || tr_x)
       throw std::logic_error("single stages run the plain step: turn the learned step and trace recording off first");
     if (in_ensemble) throw std::logic_error("the context belongs to an ensemble: step the ensemble");
+    write_nbrs();
     if (s == "prologue") k_prologue_launch();
     else if (s == "point_sources") k_sources_launch();
     else if (s == "encode") encode_launch();
@@ -1632,6 +1653,7 @@ struct Ctx : CtxBase {
   long long transfer(const std::string& name, void* host, long long count, bool up) override {
     if (up) not_in_ensemble("upload");
     if (!in_ensemble) (void)read_state();      // the host's mask parity and hierarchy index are current
+    if (up || name.rfind("nbr", 0) == 0) write_nbrs();
     void* dev = nullptr;
     long long len = 0;
     size_t esz = 0;
@@ -1672,11 +1694,8 @@ struct Ctx : CtxBase {
       if (name != "leaves") {
         const int k = name.size() == 4 ? name[3] - '0' : -1;
         if (k < 0 || k > 3) throw std::invalid_argument("unknown array " + name);
-        // the MWDG2 sweeps and the fused HWFV1 update derive neighbours from
-        // the labels: materialise them
-        if ((mwm ? !hc.limitslopes : fuse_fv1()) && len > 0)
-          launch_k((k_fill_nbrs<real>), dim3(nblk(len)), dim3(WG), 0, stream, P, (const int*)&st->n_leaves,
-                   (const int*)leaf, (const uint8_t*)leaflev, nbr[0], nbr[1], nbr[2], nbr[3]);
+        // the MWDG2 sweeps derive neighbours from the labels: materialise them
+        if (mwm && !hc.limitslopes) fill_nbrs(len);
         dev = nbr[k];
       } else {
         dev = leaf;
@@ -1724,6 +1743,7 @@ struct Ctx : CtxBase {
 
   void set_scalar(const std::string& name, double v) override {
     not_in_ensemble("set_scalar");
+    write_nbrs();
     DevState<real> s = read_state();
     if (name == "time") s.time = (real)v;
     else if (name == "dt") s.dt = (real)v;
@@ -1794,6 +1814,7 @@ struct Ctx : CtxBase {
     rebuild_all();
   }
   void rebuild_all() {
+    write_nbrs();
     MW_HIP(hipStreamSynchronize(stream));
     learn_invalidate();
     set_border_units();

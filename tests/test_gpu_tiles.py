@@ -108,3 +108,35 @@ def test_hwfv1_small_trees(case_dir, L, prec):
         assert np.array_equal(a.get("sig")[3:], b.get("sig")[3:])
         for c in ("eta0", "qx0", "qy0"):
             assert np.array_equal(a.get("A." + c), b.get("A." + c)), c
+
+
+@pytest.mark.parametrize("L,prec", [(3, "f64"), (5, "f32"), (6, "f64"), (8, "f32"), (9, "f64"), (10, "f32")])
+def test_hwfv1_update_after_whole_steps(case_dir, L, prec):
+    """The neighbour lists after whole HWFV1 steps are those of the last step's
+    leaves, whichever kernels made it: the update stage called on its own reads
+    them and gives what it gives after an emission of its own; new labels (the
+    decode called on its own) leave them alone; and uploaded lists stay as they
+    were uploaded, one after the other."""
+    import mwdg2
+    par = cases.random_case(os.path.join(str(case_dir), f"upd{L}{prec}"), L=L, seed=60 + L, solver="hwfv1",
+                            manning=0.03, t_end=50.0, wet_frac=0.5, srcs=2 if L > 3 else 0, stage=2 if L > 3 else 0)
+    with mwdg2.Simulation(par, prec) as a, mwdg2.Simulation(par, prec) as b, mwdg2.Simulation(par, prec) as c:
+        for sim in (a, b, c):
+            sim.step(3)
+        a.stage("fv1")
+        b.stage("emit")
+        nbrs = [b.get(f"nbr{k}") for k in range(4)]
+        b.stage("fv1")
+        ca, cb = a.counters(), b.counters()
+        assert ca["time"] == cb["time"] and ca["dt_next"] == cb["dt_next"] and ca["n_leaves"] == cb["n_leaves"]
+        for v in ("eta0", "qx0", "qy0"):
+            assert np.array_equal(a.get("A." + v), b.get("A." + v)), v
+        for name in ("prologue", "encode", "decode"):
+            c.stage(name)
+        for k in range(4):
+            assert np.array_equal(a.get(f"nbr{k}"), nbrs[k])
+            assert np.array_equal(c.get(f"nbr{k}"), nbrs[k])
+        for k in range(4):
+            c.set(f"nbr{k}", nbrs[(k + 1) % 4])
+        for k in range(4):
+            assert np.array_equal(c.get(f"nbr{k}"), nbrs[(k + 1) % 4])
