@@ -936,11 +936,19 @@ struct Ctx : CtxBase {
     if (!mwm) main_h = other;
   }
   // gated: the leaf emission of this step ran in k_emit_sweep1, which marks
-  // leaves at levels <= TOP_LEVEL (the top re-encode is skipped without them)
+  // leaves at levels <= TOP_LEVEL (the top re-encode is skipped without them).
+  // With quiet units the bands are the level-6 units themselves where that
+  // saves a flat launch (levels 6..10 at max_ref_lvl 12): quiet units leave
+  // both at once. Urban 4096^2 FP32, four of five units quiet: 30 us of kernels
+  // and a step of 443 us, as flat 11 and 10 and bands 5..9 33 and 449; with
+  // few quiet units 662 us a step both ways. Up to max_ref_lvl 11,
+  // without a flat launch to save, they lose (2048^2 265 -> 268 us a step, 700
+  // x 650 FP64 268 -> 279).
   void encode_scale_launch(bool gated = false) {
     const uint8_t* q = P.uquiet;                    // quiet units keep their stage-1 parents
     const int* gate = gated ? (const int*)&st->coarse_leaves : nullptr;
-    const Levels v = levels(L - 1);
+    const bool units = q && L - 1 > MRA_FLAT;
+    const Levels v = units ? Levels{UNIT_LEVEL, MRA_FLAT, UNIT_LEVEL - 2} : levels(L - 1);
     for (int level = L - 1; level > v.hi; --level)
       timed("encode_scale_level", [&] {
         launch_k((k_scale_level<real>), dim3((1 << (2 * level)) / WG), dim3(WG), 0, stream, st, hier[1],
@@ -952,8 +960,12 @@ struct Ctx : CtxBase {
                  (const uint8_t*)sig[cur], v.lo, v.hi, cnt[2], q, gate);
       });
     timed("encode_scale_top", [&] {
-      launch_k((k_scale_top<real>), dim3(1), dim3(top_threads(v.top)), 0, stream, st, hier[1],
-               (const uint8_t*)sig[cur], v.top, cnt[2], gate);
+      if (units)
+        launch_k((k_scale_top<real, true>), dim3(1), dim3(top_threads(v.top)), 0, stream, st, hier[1],
+                 (const uint8_t*)sig[cur], v.top, cnt[2], gate);
+      else
+        launch_k((k_scale_top<real>), dim3(1), dim3(top_threads(v.top)), 0, stream, st, hier[1],
+                 (const uint8_t*)sig[cur], v.top, cnt[2], gate);
     });
   }
   // alone: not after this step's stage 1 (whose kernel leaves the limiter's

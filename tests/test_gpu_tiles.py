@@ -140,3 +140,29 @@ def test_hwfv1_update_after_whole_steps(case_dir, L, prec):
             c.set(f"nbr{k}", nbrs[(k + 1) % 4])
         for k in range(4):
             assert np.array_equal(c.get(f"nbr{k}"), nbrs[(k + 1) % 4])
+
+
+@pytest.mark.parametrize("side", [None, 200])
+def test_learned_reencode_above_and_in_units(case_dir, side):
+    """max_ref_lvl 12: the stage-1 re-encode by level-6 units and, where the
+    step has leaves at levels <= 5 (a small DEM in the corner of the mesh), of
+    the levels above them: every significant parent of the stage-1 state holds
+    what the plain step's holds (1e-9: see test_learned_units_over_tiles)."""
+    import mwdg2
+    L, steps = 12, 12
+    d = os.path.join(str(case_dir), f"reenc{side}")
+    par = (cases.urban(d, L=L, t_end=100.0) if side is None else
+           cases.random_case(d, L=L, seed=71, manning=0.03, t_end=100.0, wet_frac=0.5, xsz=side, ysz=side - 40))
+    with mwdg2.Simulation(par, "f64") as ref, mwdg2.Mlp(3) as m, mwdg2.Simulation(par, "f64") as s:
+        s.set_learned(m, decide_every=4, full_every=16, threshold=2.0)
+        ref.step(steps)
+        s.step(steps)
+        sig = ref.get("sig")
+        assert np.array_equal(sig[3:], s.get("sig")[3:])
+        coarse = int(ref.get("leaves").min()) < parity_util.lvl_idx(6)
+        assert coarse == (side is not None)
+        nodes = np.flatnonzero(sig)
+        nodes = nodes[nodes >= (3 if coarse else parity_util.lvl_idx(6))]
+        for c in ("eta0", "eta1x", "qx0", "qy1y"):
+            a, b = ref.get("B." + c)[nodes], s.get("B." + c)[nodes]
+            assert float(np.max(np.abs(a - b))) <= 1e-9, c
