@@ -235,12 +235,12 @@ struct Ctx : CtxBase {
   int* tile_sums = nullptr;
   int *rev_z = nullptr, *rev_rm = nullptr;
   real* uprev = nullptr;
-  unsigned long long* maxh = nullptr;         // limiter: per-work-group largest stage-1 depths (bit patterns)
+  unsigned long long* maxh = nullptr;         // limiter: slots of the largest stage-1 depth (bit patterns), on list_n
   size_t Hp = 0;                              // node count rounded up to whole sibling groups
   real* xbuf = nullptr;                       // one coefficient as a plain array (parity transfers)
   real* red = nullptr;                        // [5][2 * leaf_grid()] next-step reduction slots
   WetList wet[2]{};                           // wet-leaf lists of the two MWDG2 stages
-  int* list_n = nullptr;                      // their counters
+  int* list_n = nullptr;                      // their counters (with the limiter maxh), zeroed by each step's prologue
   int n_stage = 0;                            // gauges (stage points)
   int* stage_codes = nullptr;
   real* rec = nullptr;                        // stage-output rows: time, depths, elevations, velocities
@@ -340,7 +340,6 @@ struct Ctx : CtxBase {
     for (int k = 0; k < 4; ++k) nbr[k] = alloc<int>(N);
     tile_sums = alloc<int>(nblk(std::max(1, N / 4), EMIT_TILE_MIN) + 4);   // read by fours
     st = alloc<DevState<real>>(1);
-    maxh = alloc<unsigned long long>(RED_SLOTS);
     red = alloc<real>((size_t)5 * 2 * RED_SLOTS);
     {
       // neutral slots (dt +inf, maxima 0): kernels that do not write a slot leave it neutral
@@ -350,7 +349,7 @@ struct Ctx : CtxBase {
       MW_HIP(hipMemcpyAsync(red, init.data(), sizeof(real) * init.size(), hipMemcpyHostToDevice, stream));
       MW_HIP(hipStreamSynchronize(stream));
     }
-    if (mwm && !hc.limitslopes) alloc_wet_lists();
+    if (mwm) alloc_wet_lists();
     for (int q = 0; q < 3; ++q) {
       cnt[q] = alloc<unsigned long long>(CNT_SLOTS);
       MW_HIP(hipMemsetAsync(cnt[q], 0, sizeof(unsigned long long) * CNT_SLOTS, stream));
@@ -869,14 +868,18 @@ struct Ctx : CtxBase {
   // The wet lists: a region holds the leaves of its share of the emission's
   // tiles (of any tile size) or of the sweeps' (256 leaves). Small grids, with
   // few appends, have 8 regions.
+  static constexpr int LIST_INTS = 2 * LIST_REGIONS * LIST_PAD;
   void alloc_wet_lists() {
-    if (list_n) return;
+    list_n = alloc<int>(LIST_INTS);
+    MW_HIP(hipMemsetAsync(list_n, 0, sizeof(int) * LIST_INTS, stream));
+    if (hc.limitslopes) {                           // no wet lists
+      maxh = reinterpret_cast<unsigned long long*>(list_n);
+      return;
+    }
     const int R = L <= 9 ? 8 : LIST_REGIONS;
     long long cap = 0;
     for (int t : {EMIT_TILE_MIN, 256, EMIT_TILE_MAX})             // the smallest hold 256 leaves, as the sweeps'
       cap = std::max(cap, (long long)nblk(nblk(std::max(1, N / 4), t), R) * 4 * t);
-    list_n = alloc<int>(2 * LIST_REGIONS * LIST_PAD);
-    MW_HIP(hipMemsetAsync(list_n, 0, sizeof(int) * 2 * LIST_REGIONS * LIST_PAD, stream));
     for (int q = 0; q < 2; ++q)
       wet[q] = {alloc<int>((size_t)R * cap), list_n + q * LIST_REGIONS * LIST_PAD, &st->wet_sum[q], (int)cap, R};
   }
@@ -973,10 +976,12 @@ struct Ctx : CtxBase {
   void stage2_launch(bool alone = false) {
     const int G = leaf_grid();
     if (hc.limitslopes) {
-      if (alone)
+      if (alone) {
+        MW_HIP(hipMemsetAsync(list_n, 0, sizeof(int) * LIST_INTS, stream));
         timed("maxh2", [&] {
           launch_k((k_maxh_stage2<real>), dim3(G), dim3(WG), 0, stream, st, P, leaves(), hier[1], zh, maxh);
         });
+      }
       timed("stage2", [&] {
         launch_k((k_stage2_limited<real>), dim3(G), dim3(WG), 0, stream, st, P, leaves(), hier[0], hier[1],
                            zh, uprev, (const unsigned long long*)maxh, red);
