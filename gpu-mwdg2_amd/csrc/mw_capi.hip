@@ -260,7 +260,7 @@ struct Ctx : CtxBase {
   int n_src = 0;
   bool issued_first = false;
   std::vector<void*> allocs;
-  // learned refinement (MWDG2, eps > 0, one MRA band of level-6 units)
+  // learned refinement (MWDG2, eps > 0, level-6 units: 7 <= max_ref_lvl <= 12)
   bool learn = false;
   MlpDev lw{};
   int l_decide = 8, l_full = 32;
@@ -753,10 +753,10 @@ struct Ctx : CtxBase {
   // work-group for every CU, large ones keep more of their neighbours inside
   // a tile. us per launch with 64 / 256 / 1024 nodes: dam break 256^2 FP64
   // 8.5 / 15 / 37, valley 1024^2 FP32 28 / 23 / 44, HWFV1 2048^2 (emit_write)
-  // 11 / 10 / 16, urban 4096^2 FP32 329 / 161 / 156; the single-group scan
-  // of the tiles' counts takes 4 us up to 4096 tiles and 24 us for 16384.
-  // The learned step's tiles hold whole level-6 units (one from
-  // max_ref_lvl 10 on).
+  // 11 / 10 / 16, urban 4096^2 FP32 329 / 161 / 156 (with 64 or 256 nodes that
+  // grid has more than EMIT_SELF_SCAN tiles, whose counts take a single-group
+  // scan of some 24 us first). The learned step's tiles hold whole level-6
+  // units (one from max_ref_lvl 10 on).
   int emit_tile() const {
     const int t = L <= 9 ? 64 : (L <= 11 ? 256 : 1024);
     return umode && L >= 10 ? 1 << (2 * (L - 1 - UNIT_LEVEL)) : t;
@@ -1462,7 +1462,7 @@ struct Ctx : CtxBase {
     MW_HIP(hipGetLastError());
   }
   // A scenario of a batched ensemble: the plain MWDG2 step without limiter,
-  // epsilon > 0, one MRA band of level-6 units, no recording.
+  // epsilon > 0, 7 <= max_ref_lvl <= 12, no recording.
   bool batchable() const override {
     return mwm && !hc.limitslopes && hc.epsilon > real(0.0) && L >= 7 && L <= 12 &&
            !rec && !cum && !learn && !tr_x && !profiling;

@@ -27,7 +27,7 @@ constexpr int LIST_REGIONS = 64, LIST_PAD = 32;
 constexpr int EMIT_SELF_SCAN = 4096;
 // Most level-6 units of the learned step that a tile of T nodes covers.
 template <int T>
-constexpr int EMIT_UNITS = T == EMIT_TILE_MIN ? 64 : (T == EMIT_TILE_MAX ? 1 : 4);
+constexpr int EMIT_UNITS = T == EMIT_TILE_MIN ? 64 : 1;
 constexpr int MAX_SRC = 4096;
 constexpr int RED_SLOTS = 4096;  // max work-groups of a leaf kernel (one reduction slot each)
 // Units of the learned step: level-6 nodes and their subtrees.
