@@ -166,3 +166,89 @@ def test_learned_reencode_above_and_in_units(case_dir, side):
         for c in ("eta0", "eta1x", "qx0", "qy1y"):
             a, b = ref.get("B." + c)[nodes], s.get("B." + c)[nodes]
             assert float(np.max(np.abs(a - b))) <= 1e-9, c
+
+
+@pytest.mark.parametrize("L,xsz,ysz,solver,prec,limit", [
+    (11, 1300, 1090, "hwfv1", "f32", False), (11, 1025, 1200, "hwfv1", "f64", False),
+    (12, 300, 260, "hwfv1", "f32", False), (11, 1100, 900, "mwdg2", "f32", True),
+    (11, 1030, 1100, "mwdg2", "f64", True)])
+def test_flat_levels(case_dir, L, xsz, ysz, solver, prec, limit):
+    """Levels from 10 on are flat launches in the encode, the decode and the
+    stage-1 re-encode: one of them (max_ref_lvl 11) and two (12, with 1024-node
+    emission tiles), for HWFV1 and for MWDG2 with the limiter, against the
+    oracle bit for bit."""
+    par = cases.random_case(os.path.join(str(case_dir), f"flat{L}{solver}{prec}"), L=L, seed=90 + L, xsz=xsz, ysz=ysz,
+                            solver=solver, manning=0.03, t_end=20.0, wet_frac=0.4, srcs=2, stage=2)
+    if limit:
+        with open(par, "a") as f:
+            f.write("limitslopes\ntol_Krivo     1\n")
+    parity_util.run_pair(par, prec, steps=3)
+
+
+def _level_of(h):
+    return np.floor(np.log2(3 * (h.astype(np.int64) - 3) + 1) / 2).astype(np.int64)
+
+
+def _part1(v):
+    v = v.astype(np.int64)
+    for s, m in ((8, 0x00FF00FF), (4, 0x0F0F0F0F), (2, 0x33333333), (1, 0x55555555)):
+        v = (v | (v << s)) & m
+    return v
+
+
+def _compact(c):
+    c = c.astype(np.int64) & 0x55555555
+    for s, m in ((1, 0x33333333), (2, 0x0F0F0F0F), (4, 0x00FF00FF), (8, 0x0000FFFF)):
+        c = (c | (c >> s)) & m
+    return c
+
+
+@pytest.mark.parametrize("solver", ["mwdg2", "hwfv1"])
+def test_scanned_tile_counts(case_dir, solver):
+    """Above 4096 emission tiles (max_ref_lvl 13) their leaf counts are scanned
+    by a launch of its own. A long thin DEM across the mesh puts leaves of every
+    level into tiles all along the list: the leaf list is the one that the mask
+    gives (in Morton order), and the neighbours are those of the finest cells
+    beside a leaf, by search in that list."""
+    import mwdg2
+    L, xsz, ysz = 13, 8000, 20
+    d = os.path.join(str(case_dir), f"scan{solver}")
+    par = cases.random_case(d, L=6, seed=5, solver=solver, manning=0.03, t_end=50.0)
+    with open(par) as f:
+        text = f.read()
+    with open(par, "w") as f:
+        f.write("\n".join(f"max_ref_lvl   {L}" if e.split()[:1] == ["max_ref_lvl"] else e
+                          for e in text.splitlines()) + "\n")
+    x = np.arange(xsz)[None, :]
+    z = (2.0 + np.sin(x / 300.0) + 0.3 * np.sin(x / 7.0) + 0.1 * cases.uniform(6, xsz * ysz).reshape(ysz, xsz))
+    cases.write_raster(os.path.join(d, "case.dem"), z, 0.0, 0.0, 1.0)
+    cases.write_raster(os.path.join(d, "case.start"), np.maximum(0.0, 2.0 - z), 0.0, 0.0, 1.0)
+    start_of = np.array([parity_util.lvl_idx(l) for l in range(L + 1)])
+    with mwdg2.Simulation(par, "f32") as s:
+        for _ in range(2):
+            s.step(2)
+            leaves, sig, c = s.get("leaves").astype(np.int64), s.get("sig"), s.counters()
+            nodes, expect = np.array([0]), []               # Morton codes of the level's nodes of the tree
+            for l in range(L + 1):
+                inner = sig[start_of[l] + nodes] != 0 if l < L else np.zeros(nodes.size, dtype=bool)
+                expect.append(start_of[l] + nodes[~inner])
+                nodes = (4 * nodes[inner][:, None] + np.arange(4)[None, :]).ravel()
+            expect = np.concatenate(expect)
+            lev = _level_of(expect)
+            first = (expect - start_of[lev]) << (2 * (L - lev))
+            order = np.argsort(first)
+            expect, lev, first = expect[order], lev[order], first[order]
+            assert c["n_leaves"] == leaves.size > 10000 and np.array_equal(leaves, expect)
+            last = first + (1 << (2 * (L - lev))) - 1
+            # tiles (64 x 64 cells) that hold a leaf's start: the strip alone lies in 8000 / 64 = 125
+            assert np.unique(first >> 12).size >= 125
+            xs, ys, xe, ye = _compact(first), _compact(first >> 1), _compact(last), _compact(last >> 1)
+            n = 1 << L
+            edge_n, edge_e = (ye == n - 1) | (ye == ysz - 1), (xe == n - 1) | (xe == xsz - 1)
+            for k, (xn, yn, border) in enumerate(((xe, ye + 1, edge_n), (xe + 1, ye, edge_e),
+                                                  (xs, ys - 1, ys == 0), (xs - 1, ys, xs == 0))):
+                m = _part1(np.clip(xn, 0, n - 1)) | (_part1(np.clip(yn, 0, n - 1)) << 1)
+                ml = np.minimum(lev, lev[np.searchsorted(first, m, side="right") - 1])
+                want = np.where(border, -1, start_of[ml] + (m >> (2 * (L - ml))))
+                assert np.array_equal(s.get(f"nbr{k}"), want), k
+            assert c["steps"] > 0 and c["nonfinite"] == 0 and 0.0 < c["dt_next"] < 10.0
