@@ -941,12 +941,12 @@ struct Ctx : CtxBase {
   // gated: the leaf emission of this step ran in k_emit_sweep1, which marks
   // leaves at levels <= TOP_LEVEL (the top re-encode is skipped without them).
   // With quiet units the bands are the level-6 units themselves where that
-  // saves a flat launch (levels 6..10 at max_ref_lvl 12): quiet units leave
-  // both at once. Urban 4096^2 FP32, four of five units quiet: 30 us of kernels
-  // and a step of 443 us, as flat 11 and 10 and bands 5..9 33 and 449; with
-  // few quiet units 662 us a step both ways. Up to max_ref_lvl 11,
-  // without a flat launch to save, they lose (2048^2 265 -> 268 us a step, 700
-  // x 650 FP64 268 -> 279).
+  // saves a flat launch (levels 6..10 at max_ref_lvl 12): quiet units and units
+  // outside the tree leave at once. us a step against flat 11 and 10 and bands
+  // 5..9: urban 4096^2 FP32 443 and 449 (four of five units quiet), 664 and 663
+  // (few quiet), 2500 x 1500 425 and 429, 2300 x 600 FP64 276 and 282. Up to
+  // max_ref_lvl 11, without a flat launch to save, they lose (2048^2 268 and
+  // 265, 700 x 650 FP64 279 and 268).
   void encode_scale_launch(bool gated = false) {
     const uint8_t* q = P.uquiet;                    // quiet units keep their stage-1 parents
     const int* gate = gated ? (const int*)&st->coarse_leaves : nullptr;
@@ -964,7 +964,7 @@ struct Ctx : CtxBase {
       });
     timed("encode_scale_top", [&] {
       if (units)
-        launch_k((k_scale_top<real, true>), dim3(1), dim3(top_threads(v.top)), 0, stream, st, hier[1],
+        launch_k((k_scale_top<real, true>), dim3(1), dim3(1024), 0, stream, st, hier[1],
                  (const uint8_t*)sig[cur], v.top, cnt[2], gate);
       else
         launch_k((k_scale_top<real>), dim3(1), dim3(top_threads(v.top)), 0, stream, st, hier[1],

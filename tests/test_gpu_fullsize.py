@@ -73,8 +73,9 @@ def urban12(tmp_path_factory):
 def test_headline_case_against_oracle(urban12, prec, steps):
     """The headline workload (urban 4096^2, max_ref_lvl 12) against the
     oracle after every step, bit for bit: masks, leaf and neighbour lists,
-    leaf coefficients, dt and time. The decode band that also counts the
-    emission tiles' leaves runs only from max_ref_lvl 12 on."""
+    leaf coefficients, dt and time. Two flat levels (10 and 11), of which the
+    decode's deepest counts the emission tiles' leaves, run only here and in
+    test_gpu_tiles.py's test_flat_levels."""
     import parity_util
     reps = parity_util.run_pair(urban12["par"], prec, steps=steps)
     assert len(reps) == steps
