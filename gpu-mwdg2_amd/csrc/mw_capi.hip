@@ -1175,12 +1175,17 @@ struct Ctx : CtxBase {
       encode_launch(true);
       counted = decode_launch(true, true);
     }
-    if (lrn() && P.uquiet)
+    if (lrn() && P.uquiet) {
       timed("learn", [&] {
-        launch_k(k_unit_quiet, dim3(nblk(N_UNITS)), dim3(WG), 0, stream, (const uint8_t*)sig[cur ^ 1],
-                 (const uint8_t*)utouch, (const uint8_t*)uwet, (const uint8_t*)uborder, uquiet,
-                 l_full_step() ? 1 : 0, lcnt + 2 * CNT_SLOTS);
+        with_tile([&](auto T) {
+          launch_k(k_quiet_and_count<T.value>, dim3(QUIET_GROUPS + emit_tiles()), dim3(WG), 0, stream,
+                   (const uint8_t*)sig[cur ^ 1], (const uint8_t*)utouch, (const uint8_t*)uwet,
+                   (const uint8_t*)uborder, uquiet, l_full_step() ? 1 : 0, lcnt + 2 * CNT_SLOTS,
+                   (const int*)&st->done, (const uint8_t*)leaflev, L, 1 << (2 * (L - 1)), tile_sums);
+        });
       });
+      counted = true;
+    }
     emit_launch(sweep, counted);
     cur ^= 1;
   }
